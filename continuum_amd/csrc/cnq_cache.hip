@@ -78,7 +78,7 @@ __global__ __launch_bounds__(64, WALK_WAVES) void bake_static_kernel(
     const float* __restrict__ tris, const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ static_items,
     const float* __restrict__ blas_cov, const float* __restrict__ xforms, const float* __restrict__ texels,
     const uint32_t* __restrict__ slot_block, float* __restrict__ static_cov, LightRect light, QueryParams p) {
-  __shared__ float s_acc[ACC_CELLS * 64];
+  __shared__ float s_acc[WALK_CELLS * 64];
   const uint32_t lane = lane_id();
   float poly[POLY_SLOTS];
   Lane L{s_acc + lane, poly, POLY_STRIDE, ACC_CELLS, 0u};
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(64, WALK_WAVES) void rebake_kernel(
     const float* __restrict__ texels, const uint32_t* __restrict__ block_slot, const float* __restrict__ static_cov,
     const uint32_t* __restrict__ dirty, const uint32_t* __restrict__ n_dirty, float* __restrict__ irradiance,
     LightRect light, QueryParams p, MovingMeshes mv) {
-  __shared__ float s_acc[ACC_CELLS * 64];
+  __shared__ float s_acc[WALK_CELLS * 64];
   const uint32_t lane = lane_id();
   float poly[POLY_SLOTS];
   Lane L{s_acc + lane, poly, POLY_STRIDE, ACC_CELLS, 0u};

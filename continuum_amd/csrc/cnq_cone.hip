@@ -43,7 +43,7 @@ __global__ __launch_bounds__(64, ONE ? 1 : WALK_WAVES) void cone_items_kernel(
     uint32_t* __restrict__ counters, uint64_t* __restrict__ work_out, uint32_t* __restrict__ work_counter,
     const uint32_t* __restrict__ order, uint32_t* __restrict__ item_cost, uint8_t* __restrict__ query_flags,
     uint64_t n_flags, QueryParams pa, ViewDesc v0) {
-  __shared__ float s_acc[ACC_CELLS * 64];
+  __shared__ float s_acc[WALK_CELLS * 64];
   __shared__ float s_poly[ONE ? POLY_SLOTS * 64 : 1];
   const uint32_t lane = lane_id();
   float poly[ONE ? 1 : POLY_SLOTS];

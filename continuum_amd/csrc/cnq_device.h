@@ -308,24 +308,27 @@ __device__ __forceinline__ bool may_touch(const Cone& c, f3 v0, f3 v1, f3 v2) {
   return true;
 }
 
-// ---- Per-query working memory: the 68-cell accumulation buffer in LDS,
-// lane-interleaved (cell s of lane l at s * 64 + l), so every access is
-// bank-conflict free whatever cell each lane touches, and 70 slots for clip
-// polygons (a 3D polygon of up to 10 vertices at slots 0-29, its clip
-// target at 30-59; 2D polygons at 30-49 and 50-69 once the 3D clip is done;
-// a splat's hull at 30-45) and the horizon-clipped quads of the weights.
-constexpr uint32_t ACC_CELLS = 68;
+// ---- Per-query working memory, in LDS and lane-interleaved (cell s of lane
+// l at s * 64 + l), so every access is bank-conflict free whatever cell each
+// lane touches: the 66-cell accumulation buffer (a row's last cell spills
+// into the next row's first two), then the polygon a draw works on, 7
+// vertices of 2 cells. 80 cells are 20,480 B a wave, an eighth of a CU's
+// 160 KB: two waves a SIMD.
+constexpr uint32_t ACC_CELLS = 66;
+constexpr uint32_t GRID_VERTS = 7;  // a window's square cut by a triangle's three edges
+constexpr uint32_t GRID_POLY = ACC_CELLS;
+constexpr uint32_t WALK_CELLS = ACC_CELLS + 2 * GRID_VERTS;
+// The rare general clips (a triangle crossing the near or the far plane, a
+// polygon outgrowing the 7 vertices, horizon-clipped quads of the weights)
+// work in 70 slots: a 3D polygon of up to 10 vertices at slots 0-29, its
+// clip target at 30-59; 2D polygons at 30-49 and 50-69 once the 3D clip is
+// done. They lie in the lane's private memory (scratch, stride 1); the cone
+// kernel's one-wave variant keeps them in LDS too (stride 64).
 constexpr uint32_t POLY_SLOTS = 70;
-// The clipper's workspace lives in the lane's private memory (scratch, cached
-// in L1/L2; consecutive slots, stride 1): only triangles that cross the
-// window, the near or the far plane use it, and keeping it out of LDS leaves
-// 17 KB of LDS per wave, so two waves fit on each SIMD. The cone kernel's
-// one-wave variant keeps it in LDS instead, lane-interleaved (stride 64):
-// 35 KB a wave, one wave per SIMD, no scratch round trips in the clips.
 constexpr uint32_t POLY_STRIDE = 1;
 constexpr uint32_t POLY_STRIDE_LDS = 64;
 // Waves per SIMD the walk kernels are compiled for (their registers are
-// limited to 256 a lane; the LDS, 17 KB a wave, allows it).
+// limited to 256 a lane; the LDS, 20 KB a wave, allows it).
 constexpr int WALK_WAVES = 2;
 constexpr uint32_t P3A = 0, P3B = 30, Q2A = 30, Q2B = 50;
 constexpr uint32_t MAX_POLY = 10;  // WGSL :11
@@ -346,6 +349,16 @@ struct Lane {
   }
   __device__ __forceinline__ float get(uint32_t cell) const { return acc[cell * 64u]; }
   __device__ __forceinline__ void set(uint32_t cell, float v) { acc[cell * 64u] = v; }
+  // Vertex i of the draw's polygon.
+  __device__ __forceinline__ f2 vert(uint32_t i) const {
+    const float* p = acc + (GRID_POLY + 2u * i) * 64u;
+    return f2{p[0], p[64]};
+  }
+  __device__ __forceinline__ void put_vert(uint32_t i, f2 v) {
+    float* p = acc + (GRID_POLY + 2u * i) * 64u;
+    p[0] = v.x;
+    p[64] = v.y;
+  }
   __device__ __forceinline__ f3 p3(uint32_t base, uint32_t i) const {
     const float* p = poly + (base + 3u * i) * pstride;
     return f3{p[0], p[pstride], p[2 * pstride]};
@@ -504,26 +517,87 @@ __device__ __forceinline__ uint32_t clip_to_grid(Lane& L, uint32_t& at, uint32_t
   return n;
 }
 
-// Vertex `k` (uniform) of a polygon held in registers.
-__device__ __forceinline__ f2 pick2(const f2 (&v)[MAX_POLY], uint32_t k) {
-  f2 r = v[0];
-#pragma unroll
-  for (uint32_t j = 1; j < MAX_POLY; j++) r = k == j ? v[j] : r;
-  return r;
+// Draws the edges of the polygon in LDS (n <= 8 vertices, the eighth in
+// `last`), in order; each next vertex is read while an edge is drawn.
+__device__ __forceinline__ void draw_poly(Lane& L, uint32_t n, f2 last, float weight) {
+  const f2 first = L.vert(0);
+  f2 a = first, b = L.vert(1);
+  for (uint32_t i = 1; i <= n; i++) {
+    const f2 ahead = i + 1u < GRID_VERTS ? L.vert(i + 1u) : last;
+    const f2 to = i < n ? b : first;
+    draw_edge(L, a, to, weight);
+    a = to;
+    b = ahead;
+  }
 }
 
-// Draws the polygon's edges in order (its vertices read in one batch).
-__device__ __forceinline__ void draw_poly(Lane& L, uint32_t at, uint32_t n, float weight) {
-  f2 v[MAX_POLY];
-#pragma unroll
-  for (uint32_t i = 0; i < MAX_POLY; i++) v[i] = L.p2(at, i < n ? i : 0u);
-  const f2 first = clamp_grid(v[0]);
-  f2 a = first;
-  for (uint32_t i = 0; i < n; i++) {
-    const f2 b = i + 1 < n ? clamp_grid(pick2(v, i + 1)) : first;
-    draw_edge(L, a, b, weight);
-    a = b;
+// A polygon the general clips left in private memory, brought to LDS; with
+// nine or ten vertices it is drawn from where it is instead (true).
+__device__ __forceinline__ bool draw_general(Lane& L, uint32_t at, uint32_t n, f2& last, float weight) {
+  if (n > GRID_VERTS + 1u) {
+    const f2 first = clamp_grid(L.p2(at, 0));
+    f2 a = first;
+#pragma unroll 1
+    for (uint32_t i = 1; i <= n; i++) {
+      const f2 b = i < n ? clamp_grid(L.p2(at, i)) : first;
+      draw_edge(L, a, b, weight);
+      a = b;
+    }
+    return true;
   }
+#pragma unroll 1
+  for (uint32_t i = 0; i < n && i < GRID_VERTS; i++) L.put_vert(i, clamp_grid(L.p2(at, i)));
+  if (n > GRID_VERTS) last = clamp_grid(L.p2(at, GRID_VERTS));
+  return false;
+}
+
+// `clip_line2` of the polygon in LDS, in place: at most N (<= 7) vertices
+// in, `bad` (and nothing changed) when it would leave more than 7 or when
+// the line crosses more than one edge each way, as only rounding can make
+// it. A convex polygon loses one run of vertices for the two crossings, so
+// the distances give a mask of kept vertices, its edges the crossings'
+// places, and only the two crossings are computed (the loop over ten vertices
+// computes one for every vertex some lane crosses at); the vertices after the
+// lost run move to their new places. Arithmetic and order are clip_line2's.
+template <uint32_t N>
+__device__ __forceinline__ uint32_t clip_line_lds(Lane& L, uint32_t n, f2 normal, float offset, bool& bad,
+                                                  bool& out_of_grid) {
+  f2 v[N];
+#pragma unroll
+  for (uint32_t k = 0; k < N; k++) v[k] = L.vert(k);
+  uint32_t in = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < N; k++) in |= offset - dot2(normal, v[k]) >= 0.0f ? 1u << k : 0u;
+  const uint32_t full = (1u << n) - 1u;
+  in &= full;
+  if (in == full || n == 0) return n;
+  if (in == 0) return 0;
+  const uint32_t next = (in >> 1) | ((in & 1u) << (n - 1u));
+  const uint32_t leave = in & ~next, enter = ~in & next;
+  const uint32_t i = (uint32_t)__builtin_ctz(leave), j = (uint32_t)__builtin_ctz(enter);
+  const bool kept0 = (in & 1u) != 0;
+  const uint32_t m = kept0 ? n + i + 2u - j : i + 2u - j;
+  if ((leave & (leave - 1u)) != 0 || m > GRID_VERTS) {
+    bad = true;
+    return n;
+  }
+  const f2 a = L.vert(i), b = L.vert(i + 1u == n ? 0u : i + 1u);
+  const f2 c = L.vert(j), d = L.vert(j + 1u == n ? 0u : j + 1u);
+  const float da = offset - dot2(normal, a), db = offset - dot2(normal, b);
+  const float dc = offset - dot2(normal, c), dd = offset - dot2(normal, d);
+  const f2 x = a + (b - a) * (da / (da - db));
+  const f2 y = d + (c - d) * (dd / (dd - dc));
+  // Vertex 0 kept: v0..vi, x, y, v(j+1)..; lost: y, v(j+1)..vi, x.
+  const uint32_t shift = kept0 ? i + 2u - j : 0u - j;
+#pragma unroll
+  for (uint32_t k = 1; k < N; k++)
+    if (k > j && k < n) L.put_vert(k + shift, v[k]);
+  L.put_vert(kept0 ? i + 1u : i - j + 1u, x);
+  L.put_vert(kept0 ? i + 2u : 0u, y);
+  const float g = (float)GRID;
+  out_of_grid = out_of_grid || x.x < 0.0f || x.y < 0.0f || x.x > g || x.y > g || y.x < 0.0f || y.y < 0.0f ||
+                y.x > g || y.y > g;
+  return m;
 }
 
 __device__ __forceinline__ bool in_window(const Cone& c, f3 v) {
@@ -634,10 +708,49 @@ __device__ __forceinline__ uint32_t general_polygon(const Cone& c, Lane& L, f3 v
   return qn;
 }
 
-// WGSL :350-451. A triangle wholly in front of the near plane, before the far
-// plane and inside the window projects to a triangle inside the grid, drawn
-// straight from registers; any other case builds its polygon in the lane's
-// workspace, and every such polygon goes through one grid clip and one draw.
+// The window's square in LDS, cut by the planes through the apex and each
+// edge of a triangle in front of the near plane (local corners l0..l2), with
+// the triangle's winding (WGSL :376-425). Returns the vertices left; `bad`
+// when general_polygon has to build it instead.
+__device__ __forceinline__ uint32_t window_polygon(const Cone& c, Lane& L, f3 l0, f3 l1, f3 l2, float su, float sv,
+                                                   bool& bad) {
+  const float g = (float)GRID;
+  const float d = dot3(l0, cross3(l1, l2));
+  if (d == 0.0f) return 0;
+  const bool ccw = d > 0.0f;
+  const float side = ccw ? 1.0f : -1.0f;
+  L.put_vert(0, f2{0.0f, 0.0f});
+  L.put_vert(1, ccw ? f2{g, 0.0f} : f2{0.0f, g});
+  L.put_vert(2, f2{g, g});
+  L.put_vert(3, ccw ? f2{0.0f, g} : f2{g, 0.0f});
+  uint32_t n = 4;
+  bool outside = false;
+#pragma unroll 1
+  for (uint32_t i = 0; i < 3; i++) {
+    const f3 p = i == 0 ? l0 : (i == 1 ? l1 : l2), q = i == 0 ? l1 : (i == 1 ? l2 : l0);
+    const f3 e = cross3(p, q);
+    const float len = len3(e);
+    if (len == 0.0f) continue;
+    const f3 k = e * (side / len);
+    const f2 normal{-k.x / su, -k.y / sv};
+    const float offset = k.x * c.w0 + k.y * c.w1 + k.z;
+    if (!(fabsf(normal.x) < 1e30f && fabsf(normal.y) < 1e30f && fabsf(offset) < 1e30f)) bad = true;
+    if (!bad) n = clip_line_lds<6>(L, n, normal, offset, bad, outside);
+  }
+  bad = bad || outside;
+  return n;
+}
+
+// WGSL :350-451. A triangle in front of the near plane and before the far
+// plane becomes a polygon of at most 7 vertices in LDS: itself projected
+// when it lies in the window, else the window's square cut by its edges. The
+// rest (a plane crossed, rounding that left the grid) is built by the general
+// clips in private memory and brought to LDS seven vertices at a time. One
+// loop then draws whatever the lanes hold. (The general clips used to take
+// every triangle that crosses the window: 8,900 cycles a round of draws on
+// the courtyard, most of them round trips to private memory and crossings
+// computed at every vertex, and 3,500 more where lanes drew whole triangles
+// beside them.)
 __device__ __forceinline__ bool rasterize(const Cone& c, Lane& L, f3 v0, f3 v1, f3 v2, float weight) {
   const float f0 = c.far_offset - dot3(c.far_normal, v0);
   const float f1 = c.far_offset - dot3(c.far_normal, v1);
@@ -645,32 +758,32 @@ __device__ __forceinline__ bool rasterize(const Cone& c, Lane& L, f3 v0, f3 v1, 
   const bool far_clip = f0 < 0.0f || f1 < 0.0f || f2_ < 0.0f;
   const float su = (float)GRID / (c.w2 - c.w0);
   const float sv = (float)GRID / (c.w3 - c.w1);
-  f3 l0{0.0f, 0.0f, 0.0f}, l1 = l0, l2 = l0;
-  uint32_t at = Q2A, qn = 0;
-  bool grid_clip = false, built = false;
-  if (!far_clip) {
-    l0 = to_local(c, v0), l1 = to_local(c, v1), l2 = to_local(c, v2);
-    if (l0.z >= NEAR && l1.z >= NEAR && l2.z >= NEAR && in_window(c, l0) && in_window(c, l1) && in_window(c, l2)) {
+  const f3 l0 = to_local(c, v0), l1 = to_local(c, v1), l2 = to_local(c, v2);
+  uint32_t n = 0;
+  bool general = far_clip || !(l0.z >= NEAR && l1.z >= NEAR && l2.z >= NEAR);
+  if (!general) {
+    if (in_window(c, l0) && in_window(c, l1) && in_window(c, l2)) {
       const f2 q0 = project(c, l0, su, sv), q1 = project(c, l1, su, sv), q2 = project(c, l2, su, sv);
-      if (in_grid(q0) && in_grid(q1) && in_grid(q2)) {
-        draw_edge(L, q0, q1, weight);
-        draw_edge(L, q1, q2, weight);
-        draw_edge(L, q2, q0, weight);
-        return true;
-      }
-      // Rounding put a corner a hair outside the grid: clip as the general path does.
-      L.put2(Q2A, 0, q0);
-      L.put2(Q2A, 1, q1);
-      L.put2(Q2A, 2, q2);
-      qn = 3;
-      grid_clip = true;
-      built = true;
+      L.put_vert(0, q0);
+      L.put_vert(1, q1);
+      L.put_vert(2, q2);
+      n = 3;
+      // (rounding can put a corner a hair outside the grid)
+      general = !(in_grid(q0) && in_grid(q1) && in_grid(q2));
+    } else {
+      n = window_polygon(c, L, l0, l1, l2, su, sv, general);
     }
   }
-  if (!built) qn = general_polygon(c, L, v0, v1, v2, far_clip, l0, l1, l2, su, sv, at, grid_clip);
-  if (grid_clip) qn = clip_to_grid(L, at, qn);
-  if (qn < 3) return false;
-  draw_poly(L, at, qn, weight);
+  f2 last{0.0f, 0.0f};
+  if (general) {
+    uint32_t at = Q2A;
+    bool grid_clip = false;
+    n = general_polygon(c, L, v0, v1, v2, far_clip, l0, l1, l2, su, sv, at, grid_clip);
+    if (grid_clip) n = clip_to_grid(L, at, n);
+    if (draw_general(L, at, n, last, weight)) return true;
+  }
+  if (n < 3) return false;
+  draw_poly(L, n, last, weight);
   return true;
 }
 

@@ -25,7 +25,7 @@ __global__ __launch_bounds__(64, WALK_WAVES) void sky_items_kernel(
     float* __restrict__ out_faces, uint64_t* __restrict__ out_full, uint64_t* __restrict__ work_out,
     const uint32_t* __restrict__ order, uint32_t* __restrict__ item_cost, uint32_t n, uint32_t w, uint32_t h,
     uint32_t tw_log2, QueryParams p, SkyParams sp) {
-  __shared__ float s_acc[ACC_CELLS * 64];
+  __shared__ float s_acc[WALK_CELLS * 64];
   const uint32_t lane = lane_id();
   float poly[POLY_SLOTS];
   Lane L{s_acc + lane, poly, POLY_STRIDE, ACC_CELLS, 0u};

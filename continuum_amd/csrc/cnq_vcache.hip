@@ -1139,7 +1139,7 @@ __global__ __launch_bounds__(64, WALK_WAVES) void vc_bake_kernel(VcArgs a, const
                                                      const uint32_t* __restrict__ blas_items,
                                                      const float* __restrict__ blas_cov, QueryParams p,
                                                      uint64_t* __restrict__ work, uint32_t* __restrict__ counters) {
-  __shared__ float s_acc[ACC_CELLS * 64];
+  __shared__ float s_acc[WALK_CELLS * 64];
   const uint32_t lane = lane_id();
   float poly[POLY_SLOTS];
   float wcov[MOVING ? BINS : 1];  // the lattice and guard walks' coverage

@@ -452,9 +452,10 @@ __device__ __forceinline__ f2 pick8(const f2 (&p)[8], uint32_t k) {
   return r;
 }
 
-// WGSL :490-512: clockwise hull of the 8 points (2D, in registers), written
-// at Q2A; returns its vertex count.
-__device__ __forceinline__ uint32_t hull8(Lane& L, const f2 (&p)[8]) {
+// WGSL :490-512: clockwise hull of the 8 points (2D, in registers), in LDS
+// (the eighth vertex, if rounding makes one, in `last`); returns its vertex
+// count.
+__device__ __forceinline__ uint32_t hull8(Lane& L, const f2 (&p)[8], f2& last) {
   uint32_t start = 0;
   f2 ps = p[0];
 #pragma unroll
@@ -468,7 +469,11 @@ __device__ __forceinline__ uint32_t hull8(Lane& L, const f2 (&p)[8]) {
   uint32_t cur = start;
   f2 pc = ps;  // p[cur]
   for (;;) {
-    L.put2(Q2A, n++, pc);
+    if (n < GRID_VERTS)
+      L.put_vert(n, pc);
+    else
+      last = pc;
+    n++;
     uint32_t next = (cur + 1) & 7u;
     f2 pn = pick8(p, next);
 #pragma unroll
@@ -496,11 +501,43 @@ __device__ __forceinline__ bool draw_hull(Lane& L, const f2 (&p)[8], float alpha
   bool inside = true;
 #pragma unroll
   for (uint32_t k = 0; k < 8; k++) inside = inside && in_grid(p[k]);
-  uint32_t n = hull8(L, p);
-  uint32_t at = Q2A;
-  if (!inside) n = clip_to_grid(L, at, n);
+  f2 last{0.0f, 0.0f};
+  uint32_t n = hull8(L, p, last);
+  if (!inside) {
+    // The four clips to the grid (WGSL :432-437: x >= 0, x <= 8, y >= 0,
+    // y <= 8), in LDS while at most 7 vertices are left, else by the general
+    // clips from where this got to.
+    const float g = (float)GRID;
+    bool bad = n > GRID_VERTS, unused = false;
+    uint32_t k = 0;
+#pragma unroll 1
+    for (; k < 4 && !bad; k++) {
+      const f2 normal{k == 0 ? -1.0f : (k == 1 ? 1.0f : 0.0f), k == 2 ? -1.0f : (k == 3 ? 1.0f : 0.0f)};
+      n = clip_line_lds<7>(L, n, normal, (k & 1u) ? g : 0.0f, bad, unused);
+      if (bad) break;
+    }
+    uint32_t at = Q2A;
+    if (bad) {
+#pragma unroll 1
+      for (uint32_t i = 0; i < n; i++) L.put2(Q2A, i, i < GRID_VERTS ? L.vert(i) : last);
+#pragma unroll 1
+      for (; k < 4; k++) {
+        const f2 normal{k == 0 ? -1.0f : (k == 1 ? 1.0f : 0.0f), k == 2 ? -1.0f : (k == 3 ? 1.0f : 0.0f)};
+        const uint32_t to = at == Q2A ? Q2B : Q2A;
+        n = clip_line2(L, at, n, normal, (k & 1u) ? g : 0.0f, to);
+        at = to;
+      }
+    }
+    if (bad) {
+      if (draw_general(L, at, n, last, alpha)) return true;
+    } else {
+      // (a crossing's other coordinate can round a hair outside)
+#pragma unroll 1
+      for (uint32_t i = 0; i < n; i++) L.put_vert(i, clamp_grid(L.vert(i)));
+    }
+  }
   if (n < 3) return false;
-  draw_poly(L, at, n, alpha);
+  draw_poly(L, n, last, alpha);
   return true;
 }
 
