@@ -57,8 +57,7 @@ __device__ __forceinline__ void uncapped_walk(Walk& w, float prefilter) {
   w.cone_work = 0;
   w.cone_cap = NONE;
   w.prefilter_bins = prefilter;
-  w.overflow = false;
-  w.truncated = false;
+  w.deep = 0;
 #pragma unroll
   for (int k = 0; k < 6; k++) w.work[k] = 0;
 }
@@ -141,7 +140,7 @@ __global__ __launch_bounds__(64, WALK_WAVES) void rebake_kernel(
       Stack st{0u, 0u, 0u};
       for (uint32_t k = 0; k < mv.n; k++) {
         const bool need = on && w.full < BINS &&
-                          may_touch_box(lc.c, f3{mv.lo[k].x, mv.lo[k].y, mv.lo[k].z}, f3{mv.hi[k].x, mv.hi[k].y, mv.hi[k].z});
+                          may_touch_box(lc.c, cone_margins(lc.c), f3{mv.lo[k].x, mv.lo[k].y, mv.lo[k].z}, f3{mv.hi[k].x, mv.hi[k].y, mv.hi[k].z});
         add_mesh_coverage<false>(x, lc.c, mv.mesh[k], need, w, st, 0, L);
       }
       uint64_t touched = 0;

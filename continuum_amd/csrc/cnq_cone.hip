@@ -79,7 +79,7 @@ __global__ __launch_bounds__(64, ONE ? 1 : WALK_WAVES) void cone_items_kernel(
     const bool valid = xpix < v.w && ypix < v.h;
     const uint64_t pixel = valid ? (uint64_t)ypix * v.w + xpix : 0;
     const float* rc = receivers + 8 * (v.recv_off + pixel);
-    const LightRect r = reinterpret_cast<const LightRect*>(lights)[v.light_off + light];
+    const LightRect* r = reinterpret_cast<const LightRect*>(lights) + v.light_off + light;
     const uint64_t q = v.out_off + (uint64_t)light * ((uint64_t)v.w * v.h) + pixel;
     const QueryOut o = evaluate_query<COUNT>(x, p, L, valid, rc, r, out_cov ? out_cov + 64 * q : nullptr, work_out);
     if (valid) {

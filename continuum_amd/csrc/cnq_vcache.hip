@@ -693,8 +693,7 @@ __device__ __forceinline__ LatticeOut lattice_ratio(const Ctx& x, const QueryPar
   w.cone_cap = NONE;
   w.prefilter_bins = p.prefilter;
   w.sky_max = false;
-  w.overflow = false;
-  w.truncated = false;
+  w.deep = 0;
 #pragma unroll
   for (int k = 0; k < 6; k++) w.work[k] = 0;
   if (uni(ballot(traced) != 0ull ? 1u : 0u)) scene_coverage<COUNT, false, false, QUEUE>(x, lc.c, traced, w, L);
@@ -749,8 +748,7 @@ __device__ __forceinline__ bool guard_touched(const Ctx& x, const QueryParams& p
   w.cone_cap = NONE;
   w.prefilter_bins = p.prefilter;
   w.sky_max = false;
-  w.overflow = false;
-  w.truncated = false;
+  w.deep = 0;
   w.stop_on_touch = true;
 #pragma unroll
   for (int k = 0; k < 6; k++) w.work[k] = 0;
@@ -1223,7 +1221,8 @@ __global__ __launch_bounds__(64, WALK_WAVES) void vc_bake_kernel(VcArgs a, const
     }
     const Skip skip{back ? t.m : NONE, back ? s.tri : NONE};
     const QueryOut o = evaluate_at<COUNT, true, QUEUE>(x, p, L, listed, s.apex, back ? toward : s.normal,
-                                                on && (!on_lattice || overflow), r, nullptr, COUNT ? work : nullptr,
+                                                on && (!on_lattice || overflow),
+                                                again(reinterpret_cast<const LightRect*>(a.lights) + l), nullptr, COUNT ? work : nullptr,
                                                 skip);
     if (COUNT) {
       const uint64_t capped = ballot(listed && o.capped);

@@ -358,14 +358,18 @@ struct Walk {
   // Sky walks (SKY) only: combine by the maximum with nearest-first order
   // (params.w bit 1, a diagnostic) instead of as independent occluders.
   bool sky_max;
-  bool overflow;   // deeper than the reference's 48 entries
-  bool truncated;  // deeper than this stack's 64 (the walk stopped)
+  uint32_t deep;  // bit 0: deeper than the reference's 48 entries; bit 1: than this stack's 64 (the walk stopped)
   // A walk that only asks whether anything meets the cone (a guard cone)
   // stops once a mesh's coverage lands in a bin: the answer is settled.
   bool stop_on_touch = false;
   uint32_t work[6];  // object nodes tested, blas nodes tested, triangles tested, triangles drawn,
                      // meshes entered, blas nodes splatted
 };
+
+// What a query's set-up puts away during its walk, beside the coverage
+// values (the normal, the spot's factor, flags), so that the walk has their
+// registers.
+constexpr uint32_t KEPT_FLOATS = 5, COV_FLOATS = BINS + KEPT_FLOATS;
 
 // A triangle the cone does not see (object, triangle in `tris`): a cache
 // texel's own, when it looks for its light below its horizon (WGSL
@@ -517,7 +521,7 @@ __device__ __forceinline__ bool draw_hull(Lane& L, const f2 (&p)[8], float alpha
       if (bad) break;
     }
     uint32_t at = Q2A;
-    if (bad) {
+    if (CNQ_RARE(bad)) {
 #pragma unroll 1
       for (uint32_t i = 0; i < n; i++) L.put2(Q2A, i, i < GRID_VERTS ? L.vert(i) : last);
 #pragma unroll 1
@@ -528,7 +532,7 @@ __device__ __forceinline__ bool draw_hull(Lane& L, const f2 (&p)[8], float alpha
         at = to;
       }
     }
-    if (bad) {
+    if (CNQ_RARE(bad)) {
       if (draw_general(L, at, n, last, alpha)) return true;
     } else {
       // (a crossing's other coordinate can round a hair outside)
@@ -541,68 +545,48 @@ __device__ __forceinline__ bool draw_hull(Lane& L, const f2 (&p)[8], float alpha
   return true;
 }
 
-// WGSL :519-574: 0 culled, 1 splatted with nothing drawn, 2 splatted and drawn, 3 descend.
-// `before_draw` runs (for this lane) just before a splat draws into the
-// accumulator, so whatever the lane still has queued goes in first.
-template <bool SKY = false, typename F>
-__device__ __forceinline__ uint32_t node_cone_test(const Cone& c, Lane& L, float prefilter_bins, f3 lo, f3 hi,
-                                                   const float* __restrict__ cov27, F&& before_draw) {
+// WGSL :519-574: 0 culled, 1 splatted with nothing drawn, 2 splatted and drawn, 3 descend;
+// 4 with `hold`: it would draw, but the lane has triangles queued that go
+// into the accumulator first.
+template <bool SKY = false>
+__device__ __forceinline__ uint32_t node_cone_test(const Cone& c, const ConeMargins& cm, Lane& L, float prefilter_bins,
+                                                   f3 lo, f3 hi, const float* __restrict__ cov27, bool hold) {
   const float g = (float)GRID;
   f2 mnv{3.4e38f, 3.4e38f}, mxv{-3.4e38f, -3.4e38f};
-  bool far_out = true, near_out = true, out_u0 = true, out_u1 = true, out_v0 = true, out_v1 = true;
-  bool below = SKY;
-  bool inside = prefilter_bins > 0.0f;
-  // The bounding-cone test first (see may_touch_box).
-  const int quick = in_bound_quick(c, lo, hi);
-  if (quick == 0) return 0;
-#pragma unroll
-  for (uint32_t k = 0; k < 8; k++) {
-    f3 corner = box_corner(lo, hi, k);
-    if (SKY && dot3(c.horizon, corner - c.apex) >= 0.0f) below = false;
-    bool in_far = c.far_offset - dot3(c.far_normal, corner) >= 0.0f;
-    if (in_far)
-      far_out = false;
-    else
-      inside = false;
-    f3 p = to_local(c, corner);
-    if (p.z >= NEAR)
-      near_out = false;
-    else
-      inside = false;
-    if (p.x - c.w0 * p.z >= 0.0f) out_u0 = false;
-    if (c.w2 * p.z - p.x >= 0.0f) out_u1 = false;
-    if (p.y - c.w1 * p.z >= 0.0f) out_v0 = false;
-    if (c.w3 * p.z - p.y >= 0.0f) out_v1 = false;
-  }
-  if (far_out || near_out || out_u0 || out_u1 || out_v0 || out_v1 || below) return 0;
-  if (quick == 2 && !in_bound(c, (lo + hi) * 0.5f, 0.5f * len3(hi - lo))) return 0;
-  if (!inside) return 3;
+  BoxQuick b;
+  uint32_t side = box_quick<SKY, true>(c, cm, lo, hi, b);
+  if (side == BOX_UNSURE) side = box_corners<SKY>(c, lo, hi);
+  if (side == BOX_OUT) return 0;
+  if (b.bound_unsure && !in_bound(c, (lo + hi) * 0.5f, 0.5f * len3(hi - lo))) return 0;
+  if (!(prefilter_bins > 0.0f) || side != BOX_INSIDE) return 3;
   // Most nodes that get here project far wider than the prefilter's bins.
-  // A bound from approximate reciprocals settles those without the exact
-  // divisions, and only where it proves the exact extent exceeds the
-  // threshold: with a = px * rcp(pz) (within 3e-7 of px / pz relative) and
-  // G = GRID * rcp(w2 - w0), every exact projection lies within
-  // 4.4e-7 * G * (U + |w0|) of G * (a - w0), U bounding |a|; so an
-  // approximate extent above the threshold by the margins below is one the
-  // exact arithmetic also finds above it, and the result is the same.
-  {
-    const float du = c.w2 - c.w0, dv = c.w3 - c.w1;
-    if (du > 0.0f && dv > 0.0f) {
-      float ulo = 3.4e38f, uhi = -3.4e38f, vlo = 3.4e38f, vhi = -3.4e38f, umag = 0.0f, vmag = 0.0f;
-#pragma unroll
-      for (uint32_t k = 0; k < 8; k++) {
-        const f3 p = to_local(c, box_corner(lo, hi, k));
-        const float r = __builtin_amdgcn_rcpf(p.z);
-        const float u = p.x * r, v = p.y * r;
-        ulo = mn(ulo, u), uhi = mx(uhi, u), vlo = mn(vlo, v), vhi = mx(vhi, v);
-        umag = mx(umag, fabsf(u)), vmag = mx(vmag, fabsf(v));
-      }
-      const float gu = g * __builtin_amdgcn_rcpf(du), gv = g * __builtin_amdgcn_rcpf(dv);
-      const float eu = (uhi - ulo) * gu * (1.0f - 1e-6f) - 2e-6f * gu * (umag * 1.000001f + fabsf(c.w0));
-      const float ev = (vhi - vlo) * gv * (1.0f - 1e-6f) - 2e-6f * gv * (vmag * 1.000001f + fabsf(c.w1));
-      if (eu > prefilter_bins * 1.000001f || ev > prefilter_bins * 1.000001f) return 3;
-    }
-  }
+  // Two opposite corners settle those: P = C + h, Q = C - h, h's signs those
+  // of right - (xc / zc) forward, along which x / z grows fastest. Their
+  // projections lie 2 (xh zc - xc zh) / (zP zQ) apart, zP = zc + zh, zQ = zc
+  // - zh. The exact extent (of the eight projections, in f32) is at least
+  // that less the rounding of both: each projected point is off by at
+  // most m (1 + U) / zmin + 1e-6 (U + |w|), U bounding |x / z| and m the
+  // bound of box_quick; twice that here covers the corners' own arithmetic
+  // too. So a difference above the threshold by this margin is one the exact
+  // arithmetic also finds above it. (Same for `up`. Signs taken from `right`
+  // alone miss the depth's part in a window far off the axis, as a near
+  // light's is from the ground, and send a bake's nodes to the exact extents:
+  // 29.4 ms for 2,874 pages against 24.0.)
+  auto wider = [&](f3 axis, float xc, float w0, float w1) {
+    const float du = w1 - w0, zc = b.local.z;
+    const float uc = xc * __builtin_amdgcn_rcpf(zc);
+    const f3 h{copysignf(b.half.x, __builtin_fmaf(-uc, c.forward.x, axis.x)),
+               copysignf(b.half.y, __builtin_fmaf(-uc, c.forward.y, axis.y)),
+               copysignf(b.half.z, __builtin_fmaf(-uc, c.forward.z, axis.z))};
+    const float xh = fdot3(axis, h), zh = fdot3(c.forward, h);
+    const float zmin = zc - fabsf(zh), zmax = zc + fabsf(zh);
+    if (!(du > 0.0f && zmin > 0.0f)) return false;
+    const float U = (fabsf(xc) + fabsf(xh)) * __builtin_amdgcn_rcpf(zmin) * 1.001f;
+    const float apart = 2.0f * __builtin_fmaf(xh, zc, -(xc * zh));
+    const float slack = 4.0f * (b.m * (1.0f + U) * zmax + 1e-6f * (U + fabsf(w0)) * (zmin * zmax));
+    return g * (apart - slack) > prefilter_bins * du * (zmin * zmax) * 1.0001f;
+  };
+  if (wider(c.right, b.local.x, c.w0, c.w2) || wider(c.up, b.local.y, c.w1, c.w3)) return 3;
   // Every corner between the near and far planes: their projections (the
   // same arithmetic the WGSL does in its corner loop, done only for nodes
   // that survive the culls). Most such nodes are too large to splat, so the
@@ -628,7 +612,7 @@ __device__ __forceinline__ uint32_t node_cone_test(const Cone& c, Lane& L, float
   if (silhouette <= 1e-30f) return 1;
   float alpha = node_front_area(cov27, v) / silhouette;
   if (alpha <= 0.0f) return 1;
-  before_draw();
+  if (hold) return 4;
   return draw_hull(L, pts, alpha) ? 2 : 1;
 }
 
@@ -679,7 +663,11 @@ __device__ __forceinline__ float triangle_weight(const Cone& c, f3 v0, f3 v1, f3
   float weight = k.weight;
   if (k.transmit > 0.0f) {
     const f3 n = cross3(v1 - v0, v2 - v0);
-    const float cos_t = fabsf(dot3(norm3(n), norm3(direction(c, 0.5f, 0.5f))));
+    // (opaque, so the direction is not worked out ahead for every mesh and
+    // held in registers: few objects transmit)
+    float half = 0.5f;
+    asm volatile("" : "+v"(half));
+    const float cos_t = fabsf(dot3(norm3(n), norm3(direction(c, half, half))));
     const float f = 0.04f + 0.96f * pow5(1.0f - cos_t);
     float passes = k.transmit * (1.0f - f);
     if (k.volume) passes *= 1.0f - f;
@@ -796,6 +784,7 @@ __device__ __forceinline__ void add_mesh_coverage(const Ctx& x, const Cone& wc, 
     c = cone_to_object(wc, x.xforms + 16 * (size_t)xform);
     weight = cover_of(x.xforms[16 * (size_t)xform + 14]);
   }
+  const ConeMargins cm = cone_margins(c);
   const uint32_t cover_skip = (SKIP && m == skip.obj) ? skip.tri : NONE;
   clear_acc(L);
   bool touched = false;
@@ -805,42 +794,64 @@ __device__ __forceinline__ void add_mesh_coverage(const Ctx& x, const Cone& wc, 
 #pragma unroll
     for (uint32_t i = 0; i < DRAW_QUEUE; i++) q.base[i] = 0, q.bits[i] = 0;
     if (root != NONE) {
-      if (base + 1 > STACK_LIMIT) {
-        w.truncated = true;
+      if (CNQ_RARE(base + 1 > STACK_LIMIT)) {
+        w.deep |= 2u;
         return;
       }
       st.put(base, root, ballot(on));
       uint32_t sp = base + 1;
+      uint32_t again_node = 0;  // a node some lanes' splat waits at (QUEUE)
+      uint64_t again_need = 0;
       for (;;) {
         if (QUEUE) {
           // Draw rounds: while a lane's queue is full (so each has room for
-          // the one leaf a step adds), and at the walk's end until every
-          // queue is empty (one place, so the drawing code is emitted once).
-          const bool end = sp <= base;
-          while (ballot(end ? q.n != 0 : q.n == DRAW_QUEUE)) draw_round(x, c, L, q, weight, touched);
+          // the one leaf a step adds), and before a splat and at the walk's
+          // end until every queue is empty (one place, so the drawing code
+          // is emitted once).
+          const bool end = sp <= base && again_need == 0;
+          while (ballot(end || again_need ? q.n != 0 : q.n == DRAW_QUEUE)) draw_round(x, c, L, q, weight, touched);
           if (end) break;
         } else if (sp <= base) {
           break;
         }
-        sp--;
-        const uint32_t n = st.node_at(sp);
-        const uint64_t need = st.mask_at(sp);
+        uint32_t n;
+        uint64_t need;
+        if (QUEUE && again_need) {
+          n = again_node;
+          need = again_need;
+          again_need = 0;
+        } else {
+          sp--;
+          n = st.node_at(sp);
+          need = st.mask_at(sp);
+        }
         bool mine = ((need >> lane_id()) & 1u) && w.cone_work < w.cone_cap;
         if (mine) w.cone_work++;
         if (!ballot(mine)) continue;
         const NodeC node = x.blas[n];
         bool descend = false;
+        uint32_t test = 0;
         if (mine) {
           if (COUNT) w.work[1]++;
-          const uint32_t test = node_cone_test<SKY>(
-              c, L, w.prefilter_bins, f3{node.lo[0], node.lo[1], node.lo[2]}, f3{node.hi[0], node.hi[1], node.hi[2]},
-              x.blas_cov + 27 * (size_t)n, [&]() {
-                if (QUEUE)
-                  while (q.n) draw_round(x, c, L, q, weight, touched);
-              });
+          test = node_cone_test<SKY>(c, cm, L, w.prefilter_bins, f3{node.lo[0], node.lo[1], node.lo[2]},
+                                     f3{node.hi[0], node.hi[1], node.hi[2]}, x.blas_cov + 27 * (size_t)n,
+                                     QUEUE && q.n != 0);
           if (test == 2) touched = true;
           if (COUNT && (test == 1 || test == 2)) w.work[5]++;
           descend = test == 3;
+        }
+        if (QUEUE) {
+          // Lanes whose splat waits take the node again once the queues are
+          // empty (not counted twice); the others have been here already.
+          const uint64_t waits = ballot(test == 4);
+          if (waits) {
+            if (test == 4) {
+              w.cone_work--;
+              if (COUNT) w.work[1]--;
+            }
+            again_node = n;
+            again_need = waits;
+          }
         }
         const uint64_t dm = ballot(descend);
         if (!dm) continue;
@@ -881,9 +892,9 @@ __device__ __forceinline__ void add_mesh_coverage(const Ctx& x, const Cone& wc, 
             }
           }
         } else {
-          if (sp + 2 > REF_STACK) w.overflow = w.overflow || descend;
-          if (sp + 2 > STACK_LIMIT) {
-            if (descend) w.truncated = true;
+          if (sp + 2 > REF_STACK) w.deep |= descend ? 1u : 0u;
+          if (CNQ_RARE(sp + 2 > STACK_LIMIT)) {
+            w.deep |= descend ? 2u : 0u;
             continue;
           }
           st.put(sp, node.a, dm);
@@ -964,7 +975,7 @@ __device__ __forceinline__ void scene_coverage(const Ctx& x, const Cone& c, bool
       bool descend = false;
       if (mine) {
         if (COUNT) w.work[0]++;
-        if (may_touch_box<SKY>(c, lo, hi)) {
+        if (may_touch_box<SKY>(c, cone_margins(c), lo, hi)) {
           const bool splatted = (node.b & NODE_NO_SPLAT) == 0 && splat_object_node<SKY>(x, c, w, n, lo, hi, L);
           descend = !splatted;
         }
@@ -995,9 +1006,9 @@ __device__ __forceinline__ void scene_coverage(const Ctx& x, const Cone& c, bool
             farc = node.a;
           }
         }
-        if (sp + 2 > REF_STACK) w.overflow = w.overflow || descend;
-        if (sp + 2 > STACK_LIMIT) {
-          if (descend) w.truncated = true;
+        if (sp + 2 > REF_STACK) w.deep |= descend ? 1u : 0u;
+        if (CNQ_RARE(sp + 2 > STACK_LIMIT)) {
+          w.deep |= descend ? 2u : 0u;
           continue;
         }
         st.put(sp, farc, dm);
@@ -1019,41 +1030,64 @@ struct QueryOut {
   bool capped, overflow, truncated;
 };
 
+// A pointer the compiler takes for another: what is read through it is read
+// again, not kept in registers since an earlier read.
+template <typename T>
+__device__ __forceinline__ const T* again(const T* p) {
+  asm volatile("" : "+v"(p));
+  return p;
+}
+
 // `active`: the lane traces (a valid query at a point that is not a sky or
-// light pixel); `skip`: the triangle this cone does not see (with SKIP).
+// light pixel); `skip`: the triangle this cone does not see (with SKIP). The
+// light, the normal and what the set-up decided are put away during the walk.
 template <bool COUNT, bool SKIP = false, bool QUEUE = false>
 __device__ __forceinline__ QueryOut evaluate_at(const Ctx& x, const QueryParams& p, Lane& L, bool valid, f3 point,
-                                                f3 normal, bool active, const LightRect& r,
+                                                f3 normal, bool active, const LightRect* __restrict__ light,
                                                 float* __restrict__ cov_out, uint64_t* __restrict__ work_out,
                                                 Skip skip = Skip{NONE, NONE}) {
   Walk w;
-  float cov[BINS];
+  float cov[COV_FLOATS];
   w.cov = cov;
 #pragma unroll
   for (uint32_t b = 0; b < BINS; b++) w.cov[b] = 0.0f;
   w.full = 0;
   w.cone_work = 0;
-  w.overflow = false;
-  w.truncated = false;
+  w.deep = 0;
   w.prefilter_bins = p.prefilter;
 #pragma unroll
   for (int k = 0; k < 6; k++) w.work[k] = 0;
 
-  const float spot = spot_falloff(r, norm3(point - light_center(r)));
-  const bool on = active && spot > 0.0f && faces_light(r, point, normal);
-  float value = 0.0f;
+  float* const kept = w.cov + BINS;
+  constexpr uint32_t ON = 1, OK = 2, WIDE_WINDOW = 4, WIDE_CLIPPED = 8;
+  Cone c{};
+  {
+    const LightRect r = *light;
+    const float spot = spot_falloff(r, norm3(point - light_center(r)));
+    const bool on = active && spot > 0.0f && faces_light(r, point, normal);
+    LightCone lc;
+    lc.ok = false;
+    lc.wide_clipped = false;
+    lc.wide_window = false;
+    lc.c = Cone{};
+    if (p.profile_stage != 1) {
+      lc = light_cone_rect(point, r, p.wide_extent);
+      w.cone_cap = lc.wide_window ? p.wide_cone_cap : p.light_cone_cap;
+    }
+    c = lc.c;
+    kept[0] = normal.x, kept[1] = normal.y, kept[2] = normal.z, kept[3] = spot;
+    kept[4] = __uint_as_float((on ? ON : 0u) | (lc.ok ? OK : 0u) | (lc.wide_window ? WIDE_WINDOW : 0u) |
+                              (lc.wide_clipped ? WIDE_CLIPPED : 0u));
+    if (p.profile_stage != 1 && p.profile_stage != 2)
+      scene_coverage<COUNT, SKIP, false, QUEUE>(x, c, on && lc.ok, w, L, skip);
+  }
+  const uint32_t flags = __float_as_uint(kept[4]);
+  const bool on = (flags & ON) != 0, ok = (flags & OK) != 0, wide_clipped = (flags & WIDE_CLIPPED) != 0;
   bool capped = false;
-  LightCone lc;
-  lc.ok = false;
-  lc.wide_clipped = false;
-  lc.wide_window = false;
   if (p.profile_stage != 1) {
-    lc = light_cone_rect(point, r, p.wide_extent);
-    const bool traced = on && lc.ok;
-    w.cone_cap = lc.wide_window ? p.wide_cone_cap : p.light_cone_cap;
-    if (p.profile_stage != 2) scene_coverage<COUNT, SKIP, false, QUEUE>(x, lc.c, traced, w, L, skip);
+    const bool traced = on && ok;
     capped = traced && w.cone_work >= w.cone_cap;
-    if (w.cone_work >= w.cone_cap && lc.wide_window && !lc.wide_clipped) {
+    if (w.cone_work >= w.cone_cap && (flags & WIDE_WINDOW) != 0 && !wide_clipped) {
 #pragma unroll
       for (uint32_t b = 0; b < BINS; b++) w.cov[b] = 1.0f;
       w.full = BINS;
@@ -1072,22 +1106,25 @@ __device__ __forceinline__ QueryOut evaluate_at(const Ctx& x, const QueryParams&
     o.touched |= (uint64_t)(w.cov[b] > 0.0f) << b;
     L.set(b, w.cov[b]);  // the coverage, for the weights' loop (the accumulator is free now)
   }
-  if (p.profile_stage != 1 && on && lc.ok) {
+  const f3 nrm = ld3(kept);
+  float value = 0.0f;
+  if (p.profile_stage != 1 && on && ok) {
+    const LightRect r = *again(light);
     if (is_sphere(r)) {
-      value = sphere_unshadowed(point, normal, r) * sphere_open_share(L, lc.c, normal, lc.wide_clipped);
+      value = sphere_unshadowed(c.apex, nrm, r) * sphere_open_share(L, c, nrm, wide_clipped);
     } else {
-      value = cone_visible(L, lc.c, normal, o.touched);
-      if (lc.wide_clipped) {
+      value = cone_visible(L, c, nrm, o.touched);
+      if (wide_clipped) {
         bool all_above;
-        const float kept = window_weight4(L, lc.c, normal, all_above);
-        value = (kept > 1e-9f ? value / kept : 1.0f) * rect_open(L, point, normal, r);
+        const float open = window_weight4(L, c, nrm, all_above);
+        value = (open > 1e-9f ? value / open : 1.0f) * rect_open(L, c.apex, nrm, r);
       }
     }
   }
-  o.visible = spot * value;
+  o.visible = kept[3] * value;
   o.capped = capped;
-  o.overflow = w.overflow;
-  o.truncated = w.truncated;
+  o.overflow = (w.deep & 1u) != 0;
+  o.truncated = (w.deep & 2u) != 0;
   if (valid && cov_out) {
 #pragma unroll
     for (uint32_t b = 0; b < BINS; b++) cov_out[b] = w.cov[b];
@@ -1109,7 +1146,7 @@ __device__ __forceinline__ QueryOut evaluate_at(const Ctx& x, const QueryParams&
 // a negative normal.w traces nothing).
 template <bool COUNT>
 __device__ __forceinline__ QueryOut evaluate_query(const Ctx& x, const QueryParams& p, Lane& L, bool valid,
-                                                   const float* __restrict__ rc, const LightRect& r,
+                                                   const float* __restrict__ rc, const LightRect* __restrict__ r,
                                                    float* __restrict__ cov_out, uint64_t* __restrict__ work_out) {
   return evaluate_at<COUNT>(x, p, L, valid, ld3(rc), ld3(rc + 4), valid && rc[7] >= 0.0f, r, cov_out, work_out);
 }
@@ -1167,8 +1204,7 @@ __device__ __forceinline__ SkyOut evaluate_sky_face(const Ctx& x, const QueryPar
   w.full = 0;
   w.cone_work = 0;
   w.cone_cap = 0xffffffffu;  // sky walks have no cap (WGSL :1059)
-  w.overflow = false;
-  w.truncated = false;
+  w.deep = 0;
   w.sky_max = sp.max_combine != 0;
   w.prefilter_bins = p.prefilter * (sp.prefilter_scale > 0.0f ? sp.prefilter_scale : 1.0f);
 #pragma unroll
