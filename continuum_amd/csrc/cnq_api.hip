@@ -241,6 +241,7 @@ cnq::ItemArgs item_args(cnq_scene* s, const float* receivers, const float* light
   a.item_cost = nullptr;
   a.query_flags = s->query_flags;
   a.n_flags = s->query_flags ? s->n_query_flags : 0;
+  a.queue = !s->instanced && s->max_leaf <= 32;
   return a;
 }
 
@@ -649,6 +650,7 @@ int cnq_irradiance_device(cnq_scene* s, const float* receivers, uint64_t n, cons
   // The receivers as an n x 1 view, tiles of 64 consecutive receivers.
   cnq::ItemArgs a = item_args(s, receivers, lights, vis, full, touched, cov);
   a.p = query_params(s, o, 64);
+  a.queue = false;  // (a list's points may lie anywhere)
   cnq::ViewDesc& v = a.v0;
   v.recv_off = 0;
   v.out_off = 0;

@@ -97,6 +97,7 @@ struct ItemArgs {
   // stack, bit 2 this build truncated it.
   uint8_t* __restrict__ query_flags;
   uint64_t n_flags;
+  bool queue;  // draw from the lanes' queues (leaves of at most 32 triangles only)
   QueryParams p;
 };
 

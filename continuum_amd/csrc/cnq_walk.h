@@ -1144,11 +1144,11 @@ __device__ __forceinline__ QueryOut evaluate_at(const Ctx& x, const QueryParams&
 
 // One query at receiver `rc` (the reference's ReceiverGpu: point, normal;
 // a negative normal.w traces nothing).
-template <bool COUNT>
+template <bool COUNT, bool QUEUE = false>
 __device__ __forceinline__ QueryOut evaluate_query(const Ctx& x, const QueryParams& p, Lane& L, bool valid,
                                                    const float* __restrict__ rc, const LightRect* __restrict__ r,
                                                    float* __restrict__ cov_out, uint64_t* __restrict__ work_out) {
-  return evaluate_at<COUNT>(x, p, L, valid, ld3(rc), ld3(rc + 4), valid && rc[7] >= 0.0f, r, cov_out, work_out);
+  return evaluate_at<COUNT, false, QUEUE>(x, p, L, valid, ld3(rc), ld3(rc + 4), valid && rc[7] >= 0.0f, r, cov_out, work_out);
 }
 
 // ---- Sky light: a uniform sky through six cube-face mask cones (WGSL
