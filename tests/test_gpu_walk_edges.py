@@ -47,6 +47,18 @@ def _check(device, meshes, recv, lights, **kw):
     assert np.array_equal(gc[ok].view(np.uint32), rc[ok].view(np.uint32)), "coverage differs"
     assert np.array_equal(gv[ok].view(np.uint32), rv[ok].view(np.uint32)), "irradiance differs"
     assert int((gt != 0).sum()) > 0
+    # The same points as a view, whose walks draw from the lanes' queues.
+    import torch
+    n, q = len(recv), len(rv)
+    scene = Scene(device, flat)
+    vis = torch.zeros(q, device="cuda:0")
+    full, touched = (torch.zeros(q, dtype=torch.int64, device="cuda:0") for _ in range(2))
+    scene.view_query_device(torch.from_numpy(recv).to("cuda:0"), n, 1, torch.from_numpy(lights).to("cuda:0"),
+                            _lib.default_options(hierarchy=2, **kw), vis, full, touched, tile_w=64)
+    torch.cuda.synchronize()
+    assert np.array_equal(full.cpu().numpy().view(np.uint64)[ok], rf[ok]), "a view's full masks differ"
+    assert np.array_equal(touched.cpu().numpy().view(np.uint64)[ok], rt[ok]), "a view's touched masks differ"
+    assert np.array_equal(vis.cpu().numpy().view(np.uint32)[ok], rv[ok].view(np.uint32)), "a view's irradiance differs"
 
 
 @pytest.mark.parametrize("offset", [0.0, 1000.0])
