@@ -21,9 +21,8 @@
 // lane as the reference's `packet_first` does; it cannot change coverage
 // (meshes combine by the maximum), only which nodes a capped walk reaches.
 //
-// Per-query state: the 64 bins' coverage in VGPRs (every access unrolled to
-// constant indices), the 68-cell accumulation buffer in LDS, interleaved by
-// lane.
+// Per-query state: the 64 bins' coverage in private memory; the 66-cell
+// accumulation buffer and a draw's polygon in LDS, interleaved by lane.
 #pragma once
 #include "cnq_kernels.h"
 
