@@ -248,19 +248,25 @@ __device__ __forceinline__ f3 box_corner(f3 lo, f3 hi, uint32_t k) {
 // 40. The corner tests are f32, so this answers only where its sum clears
 // zero by `m`, which bounds the rounding of both sides. Both start from the
 // same lo - apex and hi - apex (u = 2^-24): the corner tests' products and
-// sums add at most u |d| (4 + 5 |w|), the centre's and half extents' 4 u (1 +
-// |w|) (|D| + |H|), in all under 9 u (1 + |w|) (|D| + |H|); m takes 12 u. (The
+// sums add at most u |d| (4 + 5 |w|); the centre's part 4 u (1 + |w|) |D|; the
+// half extents' (their own rounding, the gradient's, its products and sums)
+// 6 u (1 + |w|) |H|: in all 11 u (1 + |w|) (|D| + |H|), and m takes 12 u. (The
 // tighter the better: a wave goes to the corners when any of its 64 lanes
 // has to.) The far plane's test is of world coordinates, so its margin adds
 // 8 u (|far offset| + |apex|). The bounding cone's test of the box's sphere
 // (len, r) compares axis . d with cos sqrt(len^2 - r^2) - sin r by
 // approximate square roots (1 ulp): with len^2 - r^2 >= 1e-2 len^2 both sides
-// are within 4e-6 (|cos| + |sin|) len of `in_bound`'s, whose centre is rounded
-// in world coordinates (11 u |apex| at most in the difference); the margin
-// allows 2e-5 of |d|_1 >= len and 13 u |apex|_1. What comes closer (or is not
-// a number, or an empty box) goes to the corners (BOX_UNSURE) or to
-// `in_bound` (`bound_unsure`: a cone of half a degree leaves most boxes near
-// it there, so the planes are asked first).
+// are within 4e-6 (|cos| + |sin|) len of `in_bound`'s; the margin allows 2e-5
+// of |d|_1 >= len. `in_bound` rounds the centre in world coordinates, up to
+// e = u |apex|_1 off: len^2 moves by less than `slip` = 2 s |d|_1 + s^2 with
+// s = 13 e, so a box is out of its sphere (which lets everything pass) only
+// where len^2 - r^2 exceeds that, and there the two sides move by at most
+// 1.02 e len / sqrt(len^2 - r^2) + e <= 11.2 e, of which the margin allows 13.
+// (Without `slip` there, 1 to 3 in 10^6 boxes close by an apex 10^5 m from the
+// origin are told missed though the sphere holds the apex.) What comes closer
+// (or is not a number, or an empty box) goes to the corners (BOX_UNSURE) or to
+// `in_bound` (`bound_unsure`: a cone of half a degree leaves most boxes near it
+// there, so the planes are asked first).
 // With the corners a visit of a triangle hierarchy's node took about 2,000
 // cycles (400 instructions), 1,900 of them in the tests; 20,011 scattered
 // points by 3 lights went from 7.1 to 5.5 ms, a 1280 x 720 view of the rock
@@ -308,7 +314,8 @@ __device__ __forceinline__ uint32_t box_quick(const Cone& c, const ConeMargins& 
   const float rhs = __builtin_fmaf(c.bcos, __builtin_amdgcn_sqrtf(fmaxf(t, 0.0f)),
                                    -(c.bsin * __builtin_amdgcn_sqrtf(r2)));
   const float over = fdot3(c.baxis, d) - rhs, bm = __builtin_fmaf(cm.bound, d1, cm.bound_apex);
-  const bool sized = (t > 1e-2f * l2) & (l2 > 1e-20f) & (l2 < 1e30f);
+  const float slip = cm.bound_apex * __builtin_fmaf(2.0f, d1, cm.bound_apex);
+  const bool sized = (t > __builtin_fmaf(1e-2f, l2, slip)) & (l2 > 1e-20f) & (l2 < 1e30f);
   if (sized & (over < -bm)) return BOX_OUT;
   b.local = f3{fdot3(c.right, d), fdot3(c.up, d), fdot3(c.forward, d)};
   // The least of the four window planes' largest values.
@@ -331,7 +338,7 @@ __device__ __forceinline__ uint32_t box_quick(const Cone& c, const ConeMargins& 
   bool out = (side < -mw) | (zr < -b.m) | (fr < -mf);
   bool sure = (side > mw) & (zr > b.m) & (fr > mf);
   b.bound_unsure = !((sized & (over > bm)) |
-                     ((l2 + 2.0f * cm.bound_apex * d1 < 0.9999f * r2) & (r2 > 1e-20f) & (r2 < 1e30f)) |
+                     ((l2 + slip < 0.9999f * r2) & (r2 > 1e-20f) & (r2 < 1e30f)) |
                      (c.bcos < -1.0f));
   if (SKY) {
     // (a zero horizon culls nothing)
