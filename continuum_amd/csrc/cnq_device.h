@@ -253,7 +253,10 @@ __device__ __forceinline__ f3 box_corner(f3 lo, f3 hi, uint32_t k) {
 // 6 u (1 + |w|) |H|: in all 11 u (1 + |w|) (|D| + |H|), and m takes 12 u. (The
 // tighter the better: a wave goes to the corners when any of its 64 lanes
 // has to.) The far plane's test is of world coordinates, so its margin adds
-// 8 u (|far offset| + |apex|). The bounding cone's test of the box's sphere
+// 8 u (|far offset| + |apex|). A horizon is the caller's normal, of any length:
+// its margin is m times its largest component, or m (m alone answered 78 of
+// the 3.2 million questions of a test with lengths up to 10^6 wrongly). The
+// bounding cone's test of the box's sphere
 // (len, r) compares axis . d with cos sqrt(len^2 - r^2) - sin r by
 // approximate square roots (1 ulp): with len^2 - r^2 >= 1e-2 len^2 both sides
 // are within 4e-6 (|cos| + |sin|) len of `in_bound`'s; the margin allows 2e-5
@@ -280,15 +283,17 @@ __device__ __forceinline__ f3 abs3(f3 a) { return f3{fabsf(a.x), fabsf(a.y), fab
 __device__ __forceinline__ float sum3(f3 a) { return a.x + a.y + a.z; }
 
 // A cone's part of the tests: the far plane seen from the apex and its
-// margin, the window's factor, the bounding cone's margins.
+// margin, the window's factor, the bounding cone's margins, the horizon's
+// factor (sky walks).
 struct ConeMargins {
-  float far, far_margin, window, bound, bound_apex;
+  float far, far_margin, window, bound, bound_apex, horizon;
 };
 __device__ __forceinline__ ConeMargins cone_margins(const Cone& c) {
   const float apex = sum3(abs3(c.apex));
   return ConeMargins{c.far_offset - fdot3(c.far_normal, c.apex), 4.8e-7f * (fabsf(c.far_offset) + apex),
                      1.0f + fmaxf(fmaxf(fabsf(c.w0), fabsf(c.w1)), fmaxf(fabsf(c.w2), fabsf(c.w3))),
-                     2e-5f * (fabsf(c.bcos) + fabsf(c.bsin)), 7.8e-7f * apex};
+                     2e-5f * (fabsf(c.bcos) + fabsf(c.bsin)), 7.8e-7f * apex,
+                     fmaxf(fmaxf(1.0f, fabsf(c.horizon.x)), fmaxf(fabsf(c.horizon.y), fabsf(c.horizon.z)))};
 }
 
 // The box in the cone's frame: its centre there, half extents (world) and m.
@@ -343,8 +348,9 @@ __device__ __forceinline__ uint32_t box_quick(const Cone& c, const ConeMargins& 
   if (SKY) {
     // (a zero horizon culls nothing)
     const float hr = fdot3(c.horizon, d) + fdot3(abs3(c.horizon), b.half);
-    out = out | (hr < -b.m);
-    sure = sure & ((hr > b.m) | ((c.horizon.x == 0.0f) & (c.horizon.y == 0.0f) & (c.horizon.z == 0.0f)));
+    const float mh = b.m * cm.horizon;
+    out = out | (hr < -mh);
+    sure = sure & ((hr > mh) | ((c.horizon.x == 0.0f) & (c.horizon.y == 0.0f) & (c.horizon.z == 0.0f)));
   }
   uint32_t r = BOX_CROSS;
   if (INSIDE) {

@@ -104,3 +104,26 @@ def test_sky_faces_over_touching_boxes_match_the_oracle(device, prefilter):
     assert np.array_equal(np.asarray(full).ravel(), np.asarray(rfull).ravel()), "full masks differ"
     assert np.array_equal(faces.ravel().view(np.uint32), np.asarray(rfaces, np.float32).ravel().view(np.uint32))
     assert np.array_equal(out.view(np.uint32), np.asarray(ro, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("length", [1e-3, 100.0, 1e5])
+def test_sky_normals_of_any_length_match_the_oracle(device, length):
+    """A receiver's normal is taken as it comes: its horizon's plane runs
+    along the faces of boxes and through the corners of a tilted grid."""
+    rng = np.random.default_rng(11)
+    boxes = [box_mesh([x, y, z], [x + 1, y + 1, z + 1]) for x, y, z in ((1, 0, 0), (-2, 1, -1), (0, -3, 1), (2, 2, -2))]
+    n = np.array([0.36, 0.48, 0.8])
+    u, v = np.array([0.8, -0.6, 0.0]), np.cross(n, [0.8, -0.6, 0.0])
+    flats = np.array([[3 * a * u + 3 * b * v + k * 1e-7 * n for a, b, k in ((i, j, 1), (i + 1, j, -1), (i, j + 1, 0))]
+                      for i in range(-2, 2) for j in range(-2, 2)], np.float32)
+    meshes = boxes + [flats, _soup(rng, 200, 0.2, [-3, -3, -3], [3, 3, 3])]
+    points = [[0, 0, 0], [0, 0, 1], [1, 1, 1], [0.5, -0.5, 0.25], [2, 2, -1]]
+    recv = receivers_array([[*p, *(length * np.asarray(d, np.float64))] for p in points
+                            for d in (n, [0, 0, 1], [0, 1, 0], [0.6, 0, 0.8], -n)])
+    flat = Flat.build_arrays(*meshes_to_arrays(meshes))
+    opts = dict(hierarchy=2, prefilter=1.0)
+    out, faces, full = Scene(device, flat).sky(recv, _lib.default_options(**opts))
+    ro, rfaces, rfull, *_ = O.sky(flat, recv, O.opts_array(**opts))
+    assert np.array_equal(np.asarray(full).ravel(), np.asarray(rfull).ravel()), "full masks differ"
+    assert np.array_equal(faces.ravel().view(np.uint32), np.asarray(rfaces, np.float32).ravel().view(np.uint32))
+    assert np.array_equal(out.view(np.uint32), np.asarray(ro, np.float32).view(np.uint32))

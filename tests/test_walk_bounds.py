@@ -42,6 +42,12 @@ def test_boxes_are_settled_as_by_their_corners(walk_bounds, mode, count, seed):
     assert settled > cases / 4  # (two checks a box: the short cut did settle boxes)
 
 
+def test_sky_boxes_are_settled_by_the_horizon_of_any_normal(walk_bounds):
+    """Normals of length 1 and of 10^-3 to 10^6, boxes with corners in the horizon's plane."""
+    cases, settled = walk_bounds("sky", 200000, 1)
+    assert settled > cases / 4
+
+
 @pytest.mark.parametrize("mode,count", [("triangle", 200000), ("hull", 500000)])
 def test_draws_are_the_general_clips(walk_bounds, mode, count):
     cases, settled = walk_bounds(mode, count, 3)
