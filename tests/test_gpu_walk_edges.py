@@ -127,3 +127,51 @@ def test_sky_normals_of_any_length_match_the_oracle(device, length):
     assert np.array_equal(np.asarray(full).ravel(), np.asarray(rfull).ravel()), "full masks differ"
     assert np.array_equal(faces.ravel().view(np.uint32), np.asarray(rfaces, np.float32).ravel().view(np.uint32))
     assert np.array_equal(out.view(np.uint32), np.asarray(ro, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("cap", [150, 190, 233, 300])
+def test_a_waiting_splat_counts_once_against_the_node_cap(device, cap):
+    """One mesh (whose children's order is fixed) of small clusters that
+    splat and larger triangles that are drawn, under a small cap: a lane whose
+    splat waits for its queued triangles takes the node again, and still stops
+    where the list's walk (no queue) and the oracle's stop, at every query."""
+    import torch
+    rng = np.random.default_rng(17)
+    clusters = (rng.uniform([-1, -1, 0.5], [1, 1, 3], (80, 1, 1, 3)) + rng.uniform(-0.02, 0.02, (80, 12, 1, 3)) +
+                rng.uniform(-0.02, 0.02, (80, 12, 3, 3))).reshape(-1, 3, 3)
+    mesh = np.concatenate([clusters.astype(np.float32), _soup(rng, 150, 0.25, [-1, -1, 0.5], [1, 1, 3])])
+    flat = Flat.build_arrays(*meshes_to_arrays([mesh]))
+    recv = receivers_array(np.concatenate([rng.uniform([-1, -1, -0.5], [1, 1, 0.5], (700, 3)),
+                                           np.tile([0.0, 0.0, 1.0], (700, 1))], 1))
+    lights = np.stack([rect_light([-0.5, 0.5, 4.0], [1, 0, 0], [0, -1, 0], one_sided=True),
+                       sphere_light([0.3, 0.2, 5.0], 0.3)])
+    kw = dict(hierarchy=2, prefilter=2.0, light_cone_cap=cap, wide_cone_cap=cap)
+    opts = _lib.default_options(**kw)
+    rv, rf, rt, _, capped, _ = O.irradiance(flat, recv, lights, O.opts_array(**kw))
+    assert 0 < int(capped.sum()) < len(capped)
+    scene = Scene(device, flat)
+    n, q = len(recv), len(rv)
+    flags = torch.zeros(q, dtype=torch.uint8, device="cuda:0")
+    scene.set_query_flags(flags)
+    r, l = torch.from_numpy(recv).to("cuda:0"), torch.from_numpy(lights).to("cuda:0")
+    for name in ("view", "list"):
+        vis = torch.zeros(q, device="cuda:0")
+        full, touched = (torch.zeros(q, dtype=torch.int64, device="cuda:0") for _ in range(2))
+        flags.zero_()
+        if name == "view":
+            scene.view_query_device(r, n, 1, l, opts, vis, full, touched, tile_w=64)
+        else:
+            scene.query_device(r, l, opts, vis, full, touched)
+        torch.cuda.synchronize()
+        assert np.array_equal(flags.cpu().numpy() & 1, capped), f"{name}: other queries stop at the cap"
+        assert np.array_equal(full.cpu().numpy().view(np.uint64), rf), f"{name}: full masks differ"
+        assert np.array_equal(touched.cpu().numpy().view(np.uint64), rt), f"{name}: touched masks differ"
+        assert np.array_equal(vis.cpu().numpy().view(np.uint32), rv.view(np.uint32)), f"{name}: irradiance differs"
+    scene.set_query_flags(None)
+    # Both splats and triangles drawn, several a query.
+    scene.set_count_work(True)
+    scene.query_device(r, l, opts, vis, full, touched)
+    torch.cuda.synchronize()
+    work = scene.counters()[1]
+    scene.set_count_work(False)
+    assert min(int(work[3]), int(work[5])) > q, work
