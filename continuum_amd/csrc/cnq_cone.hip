@@ -135,13 +135,23 @@ void launch_items_variant(const ItemArgs& a, bool count_work, uint32_t persisten
 // or with `waves` 1 the one-wave variant (workspace in LDS), for launches
 // without the work counters that walk both hierarchies unprofiled. With
 // `a.queue` the lanes' triangles are drawn from queues: item_args asks for it
-// over scenes of plain meshes whose leaves hold at most 32 triangles, where a
-// mesh's walk crosses many leaves (the rock field's 1280 x 720 view 6.77 ms
-// against 7.82 drawing leaf by leaf, the courtyard frame 62.0 against 63.1,
-// a batch of 5 courtyard views 134.8 against about 139). Instanced objects
-// (a few leaves each: the boulder view 42.8 ms against 41.0) and lists, whose
-// scattered points draw one lane at a time either way (20,011 points 6.11 ms
-// against 5.49), draw leaf by leaf.
+// over scenes of plain meshes whose leaves hold at most 32 triangles. The
+// counted and the one-wave variants always draw leaf by leaf (the counts are
+// the same; a tuner that tries one wave tries that drawing with it).
+// Queued against leaf by leaf, one build, in turn, 1280 x 720 x 3 lights:
+// rounded meshes of 250 leaves and more gain (the rock field 4.56 ms against
+// 4.72, over five cameras 0.76-0.98 of the time; 3,000 spheres of 1,280
+// triangles 20.7 against 22.7), meshes of up to 64 leaves gain or lose a few
+// percent by how much of a cone they fill (3,000 spheres of 320 triangles
+// 10.5 against 11.0, 300 of them 3.79 against 3.71, 300 boxes 2.17 against
+// 2.18), and rooms lose where little is drawn (a 256 x 256 room view 0.99-1.08
+// of the time, the courtyard from one camera 52.4 against 50.5) or come out
+// even (its frames 0.99-1.03, batches of 5 views 0.88-1.07). Neither a mesh's
+// leaves nor a scene's triangles tell these apart. Instanced objects measure
+// as plain ones do near the camera (300 spheres of 9,680 triangles 13.9
+// against 14.9), but views far over a million boulders take 1.00-1.13 of the
+// time, so they draw leaf by leaf; so do lists, whose scattered points draw
+// one lane at a time either way (20,011 points by 3 lights 6.25 ms against 5.50).
 hipError_t launch_cone_items(const ItemArgs& a, bool count_work, uint32_t persistent_blocks, hipStream_t stream,
                              uint32_t waves) {
   if (a.p.n_items <= a.p.item_begin) return hipSuccess;

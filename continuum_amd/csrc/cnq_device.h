@@ -855,8 +855,9 @@ __device__ __forceinline__ uint32_t window_polygon(const Cone& c, Lane& L, f3 l0
 // plane becomes a polygon of at most 7 vertices in LDS: itself projected
 // when it lies in the window, else the window's square cut by its edges. The
 // rest (a plane crossed, rounding that left the grid) is built by the general
-// clips in private memory and brought to LDS seven vertices at a time. One
-// loop then draws whatever the lanes hold. (The general clips used to take
+// clips in private memory and, up to eight vertices of it, brought to LDS (the
+// eighth in registers; nine or ten are drawn from where they are). One loop
+// then draws whatever the lanes hold. (The general clips used to take
 // every triangle that crosses the window: 8,900 cycles a round of draws on
 // the courtyard, most of them round trips to private memory and crossings
 // computed at every vertex, and 3,500 more where lanes drew whole triangles

@@ -1222,8 +1222,8 @@ __global__ __launch_bounds__(64, WALK_WAVES) void vc_bake_kernel(VcArgs a, const
     const Skip skip{back ? t.m : NONE, back ? s.tri : NONE};
     const QueryOut o = evaluate_at<COUNT, true, QUEUE>(x, p, L, listed, s.apex, back ? toward : s.normal,
                                                 on && (!on_lattice || overflow),
-                                                again(reinterpret_cast<const LightRect*>(a.lights) + l), nullptr, COUNT ? work : nullptr,
-                                                skip);
+                                                again(reinterpret_cast<const LightRect*>(a.lights) + l), nullptr,
+                                                COUNT ? work : nullptr, skip);
     if (COUNT) {
       const uint64_t capped = ballot(listed && o.capped);
       if (lane == 0 && capped) atomicAdd(&counters[0], (uint32_t)__builtin_popcountll(capped));
