@@ -250,6 +250,41 @@ static void apex_boxes(uint64_t n) {
   }
 }
 
+// Cones of any window and far plane (a lattice cone's is its light's, not its
+// forward axis), at any scale, and boxes that are points, empty, unbounded or
+// not a number.
+static void any_boxes(uint64_t n) {
+  for (uint64_t i = 0; i < n; i++) {
+    Cone c{};
+    c.apex = any3(spread(1e-6, 1e8));
+    c.forward = unit3();
+    c.right = norm3(cross3(c.forward, unit3()));
+    c.up = cross3(c.forward, c.right);
+    const float u = (float)(uniform(-1, 1) * spread(1e-3, 1e4)), v = (float)(uniform(-1, 1) * spread(1e-3, 1e4));
+    const float eu = (float)spread(1e-6, 1e2), ev = (float)spread(1e-6, 1e2);
+    c.w0 = u - eu, c.w2 = u + eu, c.w1 = v - ev, c.w3 = v + ev;
+    c.far_normal = below(2) ? c.forward : unit3();
+    const double far = spread(1e-6, 1e8);
+    c.far_offset = dot3(c.far_normal, c.apex) + (float)far;
+    bound_cone(c, norm3(direction(c, 0.5f, 0.5f)));
+    for (int k = 0; k < 8; k++) {
+      f3 lo, hi;
+      any_box(c, below(2) ? far : spread(1e-8, 1e12), false, lo, hi);
+      switch (below(40)) {
+        case 0: hi.x = INFINITY; break;
+        case 1: lo.y = -INFINITY, hi.y = INFINITY; break;
+        case 2: hi = lo; break;
+        case 3: lo = f3{3.4e38f, 3.4e38f, 3.4e38f}, hi = -lo; break;
+        case 4: hi.z = NAN; break;
+        case 5: lo.x = -1e38f, hi.x = 1e38f; break;
+        case 6: lo = hi = c.apex; break;
+        default: break;
+      }
+      check_box<false>(c, lo, hi);
+    }
+  }
+}
+
 // ---- draws: the accumulator after a draw in LDS and after the general clips
 static void note_draw(bool a, bool b, Lanes& x, Lanes& y) {
   cases++;
@@ -338,6 +373,8 @@ int main(int argc, char** argv) {
     sky_boxes(n);
   else if (!std::strcmp(mode, "apex"))
     apex_boxes(n);
+  else if (!std::strcmp(mode, "any"))
+    any_boxes(n);
   else if (!std::strcmp(mode, "triangle"))
     triangles(n);
   else if (!std::strcmp(mode, "hull"))

@@ -33,11 +33,12 @@ def walk_bounds(tmp_path_factory):
 
 
 @pytest.mark.parametrize("seed", [1, 2])
-@pytest.mark.parametrize("mode,count", [("light", 200000), ("object", 100000), ("apex", 200000)])
+@pytest.mark.parametrize("mode,count", [("light", 200000), ("object", 100000), ("apex", 200000), ("any", 100000)])
 def test_boxes_are_settled_as_by_their_corners(walk_bounds, mode, count, seed):
     """Light cones, the same in a turned and scaled object's space, and boxes
     by an apex up to 10^6 m from the origin, where the bounding sphere's centre
-    is rounded by more than the box is wide."""
+    is rounded by more than the box is wide; cones of any window and far plane
+    over boxes that may be empty, unbounded or not a number."""
     cases, settled = walk_bounds(mode, count, seed)
     assert settled > cases / 4  # (two checks a box: the short cut did settle boxes)
 
